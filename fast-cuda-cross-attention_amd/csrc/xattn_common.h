@@ -118,6 +118,16 @@ __device__ inline const T* uniform_ptr(const T* p) {
     return (const T*)(((unsigned long long)hi << 32) | lo);
 }
 
+// uniform_ptr as the source base of dma16_m0: a v_readfirstlane's result may be
+// read by a vector memory instruction only five wait states later, which the
+// compiler keeps for its own instructions but not for inline assembly.
+template <typename T>
+__device__ inline const T* dma_base(const T* p) {
+    const T* u = uniform_ptr(p);
+    asm volatile("s_nop 4" : "+s"(u));
+    return u;
+}
+
 // 16-byte global -> LDS DMA for one lane.  The 64 lanes of the wave land at
 // lds_base + 16 * lane (lds_base must be wave-uniform).
 __device__ inline void dma16(const void* gptr, void* lds_base) {

@@ -686,6 +686,16 @@ bool launch_flash_f32(int ds, const float* Q, const float* K, const float* V, fl
         set_error(XATTN_ERR_INVALID_VALUE, "flash_f32: column parts %d not in {1, 2, 4}", ds);
         return false;
     }
+    if (ds == 4) {
+        // 16-latent workgroups: the sliced form for longer key ranges.  Its
+        // loop is 7 % faster per tile, its first tiles cost more: ranges of 7
+        // tiles measured 1.2 % slower with it, of 11 / 16 / 49 tiles 3.5 / 4.2
+        // / 6.8 % faster (B=1 NL=512, B=3 NL=197, B=1 NL=256, B=8 NL=512).
+        constexpr int kSliceMinTiles = 9;
+        const int keys = po ? (chunk < NI ? chunk : NI) : NI;
+        if ((keys + f32::BN - 1) / f32::BN >= kSliceMinTiles)
+            return launch_slice_f32(Q, K, V, out, po, pm, pl, B, NL, NI, S, chunk, stream);
+    }
     f32::Params p;
     p.Q = Q; p.K = K; p.V = V; p.out = out; p.po = po; p.pm = pm; p.pl = pl;
     p.B = B; p.NL = NL; p.NI = NI; p.S = S; p.chunk = chunk;

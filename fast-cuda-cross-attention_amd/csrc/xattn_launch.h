@@ -23,6 +23,11 @@ int f32_row_blocks(int NL, int ds);
 bool launch_flash_f32(int ds, const float* Q, const float* K, const float* V, float* out, float* po,
                       float* pm, float* pl, int B, int NL, int NI, int S, int chunk,
                       hipStream_t stream);
+// The ds = 4 form for longer key ranges (16-latent workgroups whose wavefronts
+// own column slices, xattn_slice_f32.hip).
+bool launch_slice_f32(const float* Q, const float* K, const float* V, float* out, float* po,
+                      float* pm, float* pl, int B, int NL, int NI, int S, int chunk,
+                      hipStream_t stream);
 // The LSE merge of split partials into out; parts <= 0 takes
 // lse_combine_parts' column parts (1, 2 or 4 workgroups per row; any choice
 // gives bit-identical output).
