@@ -343,7 +343,9 @@ int plan_splits(int B, int NL, int NI, int cu, int bm, int tile) {
 // the LSE merge, 10.67 µs + 0.36 µs per MB of partials written and read back,
 // + 0.08 µs per split while there are fewer merge rows (B * N_latent) than
 // CUs.  Its choice is the fastest timed plan at 27 of the 31 shapes, 0.48 %
-// slower on average and 4.4 % at worst.
+// slower on average and 4.4 % at worst.  Ranges of nine or more tiles have since
+// got faster at 16 latents (1.40-1.45 µs per tile, xattn_slice_f32.hip), which
+// the fit does not hold.
 static double f32_cost(int B, int NL, int cu, int ds, long long S, long long ct) {
     const double tile_us = ds == 1 ? 5.620 : ds == 2 ? 2.986 : 1.716;
     const long long W = (long long)B * f32_row_blocks(NL, ds) * S;

@@ -24,7 +24,8 @@
 // workgroup covers 32 or 16 latents); after QK each writes its share of S^T
 // to LDS and, after the next barrier, every wavefront of the block adds the
 // DS shares in the same order before its softmax.  The launch planner picks
-// the form and the key splits (xattn_abi.hip, f32_plan).
+// the form and the key splits (xattn_abi.hip, f32_plan); 16-latent workgroups
+// over longer key ranges run xattn_slice_f32.hip instead (launch_flash_f32).
 //
 // K and V tiles are shared by the 4 wavefronts through LDS and arrive by
 // global->LDS DMA (16 B per lane, 1 KiB per wave instruction).  Phases
