@@ -118,14 +118,22 @@ __device__ inline const T* uniform_ptr(const T* p) {
     return (const T*)(((unsigned long long)hi << 32) | lo);
 }
 
-// uniform_ptr as the source base of dma16_m0: a v_readfirstlane's result may be
-// read by a vector memory instruction only five wait states later, which the
-// compiler keeps for its own instructions but not for inline assembly.
-template <typename T>
-__device__ inline const T* dma_base(const T* p) {
-    const T* u = uniform_ptr(p);
+// Wave-uniform source address of the inline-assembly DMAs below, which take no
+// other.  A vector memory instruction may read an SGPR that a vector
+// instruction wrote (uniform_ptr's v_readfirstlane) only five wait states
+// later; the compiler keeps that for its own instructions but not for inline
+// assembly, and a DMA that comes sooner reads from a wrong address.  dma_base
+// waits them out, once per base; an offset (wave-uniform) is added by scalar
+// instructions, whose results may be read at once.  tests/test_dma_hazard.py
+// looks the compiled kernels over.
+struct DmaSrc {
+    const char* p;
+    __device__ DmaSrc operator+(size_t bytes) const { return DmaSrc{p + bytes}; }
+};
+__device__ inline DmaSrc dma_base(const void* p) {
+    const char* u = uniform_ptr((const char*)p);
     asm volatile("s_nop 4" : "+s"(u));
-    return u;
+    return DmaSrc{u};
 }
 
 // 16-byte global -> LDS DMA for one lane.  The 64 lanes of the wave land at
@@ -140,7 +148,7 @@ __device__ inline unsigned lds_u32(const void* p) {
     return (unsigned)(uintptr_t)((const __attribute__((address_space(3))) char*)p);
 }
 
-// The same DMA issued as inline assembly: lane i reads sbase + voff_i (sbase
+// The same DMA issued as inline assembly: lane i reads src + voff_i (src
 // wave-uniform, in SGPRs) and writes LDS bytes [lds_byte + 16 i, +16).  The
 // compiler does not see it, so it inserts no vmcnt waits of its own before
 // later LDS reads (it drains every outstanding DMA before a transposing LDS
@@ -148,7 +156,7 @@ __device__ inline unsigned lds_u32(const void* p) {
 // the caller orders it with wait_vmcnt + lds_barrier, which count it like any
 // vector memory load.  M0 (reserved to the compiler) is saved and restored
 // around the load and written one wait state before the load reads it.
-__device__ inline void dma16_untracked(const void* sbase, unsigned voff, unsigned lds_byte) {
+__device__ inline void dma16_untracked(DmaSrc src, unsigned voff, unsigned lds_byte) {
     unsigned saved;
     asm volatile(
         "s_mov_b32 %0, m0\n\t"
@@ -157,7 +165,7 @@ __device__ inline void dma16_untracked(const void* sbase, unsigned voff, unsigne
         "global_load_lds_dwordx4 %1, %2\n\t"
         "s_mov_b32 m0, %0"
         : "=&s"(saved)
-        : "v"(voff), "s"(sbase), "s"(lds_byte)
+        : "v"(voff), "s"(src.p), "s"(lds_byte)
         : "memory");
 }
 
@@ -168,13 +176,13 @@ __device__ inline void dma16_untracked(const void* sbase, unsigned voff, unsigne
 // destination alike, so lds_byte is the destination minus OFF.  The one wait
 // state between the write of M0 and the load is the s_nop.
 template <int OFF>
-__device__ inline void dma16_m0(const void* sbase, unsigned voff, unsigned lds_byte) {
+__device__ inline void dma16_m0(DmaSrc src, unsigned voff, unsigned lds_byte) {
     static_assert(OFF >= 0 && OFF < 4096, "global instruction offset range");
     asm volatile(
         "s_nop 0\n\t"
         "global_load_lds_dwordx4 %0, %1 offset:%3"
         :
-        : "v"(voff), "s"(sbase), "{m0}"(lds_byte), "i"(OFF)
+        : "v"(voff), "s"(src.p), "{m0}"(lds_byte), "i"(OFF)
         : "memory");
 }
 

@@ -293,8 +293,9 @@ void flash16_kernel(Params p) {
             doffv[t] = chunk_offset(t < CPWV ? CPWV * w + t : CHUNKSV - 1, LROWV / 16, DWC / 8);
     }
     const unsigned lds0 = lds_u32(lds);
+    const DmaSrc Ks = dma_base(Kb), Vs = dma_base(Vb);
     struct Dma {
-        const char* src;
+        DmaSrc src;
         unsigned m0;
     };
     auto dma_setup = [&](int ph) {
@@ -304,7 +305,7 @@ void flash16_kernel(Params p) {
         // per-lane copy would hold VGPRs across the tile loop)
         const int row0 = __builtin_amdgcn_readfirstlane(tile * BN - row_lo(tile));
         Dma d;
-        d.src = uniform_ptr(((ph & 1) ? Vb : Kb) + (size_t)row0 * ROWB);
+        d.src = ((ph & 1) ? Vs : Ks) + (size_t)row0 * ROWB;
         d.m0 = lds0 + (unsigned)((ph % NBUF) * BUFB);
         return d;
     };
@@ -352,7 +353,7 @@ void flash16_kernel(Params p) {
         // Latents past NL repeat the last one.
         constexpr int QCH = BM * (LROW / 16) / kWave;  // 1 KiB chunks of the block
         static_assert(QCH * 1024 == BM * LROW && BM * LROW <= 2 * BUFB, "Q staging");
-        const char* qsrc = uniform_ptr((const char*)(p.Q + ((size_t)b * p.NL + q0) * kDim));
+        const DmaSrc qsrc = dma_base(p.Q + ((size_t)b * p.NL + q0) * kDim);
         const int qrows = p.NL - q0;  // >= 1
         for (int m = w; m < QCH; m += NW) {
             const int u = kWave * m + lane;

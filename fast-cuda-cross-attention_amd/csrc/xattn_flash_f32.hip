@@ -222,8 +222,7 @@ void flash_f32_kernel(Params p) {
     const unsigned lds0 = lds_u32(lds);
     const int r0 = w * (CPW / ROW_CHUNKS);
     const unsigned lane16 = 16u * lane;
-    const float* const Ks = uniform_ptr(Kb);
-    const float* const Vs = uniform_ptr(Vb);
+    const DmaSrc Ks = dma_base(Kb), Vs = dma_base(Vb);
     const int nk = k1 - k0;
     auto win = [&](int n0) {  // n0 = k0 + 16 t
         return nk >= BN ? min(n0, k1 - BN) : n0;
@@ -236,7 +235,7 @@ void flash_f32_kernel(Params p) {
     // Chunk t of a phase whose window starts at src (wave-uniform) and whose
     // LDS buffer starts at byte lds_buf; chunk c of a row adds c KiB to the
     // row's source and LDS addresses (the instruction's immediate).
-    auto dma_chunk = [&](const char* src, unsigned lds_buf, int t) {
+    auto dma_chunk = [&](DmaSrc src, unsigned lds_buf, int t) {
         const int r = t / ROW_CHUNKS, c = t % ROW_CHUNKS;
         const unsigned row_lds = lds_buf + 4u * (unsigned)((r0 + r) * ROW);
         if (c == 0) dma16_m0<0>(src, voff[r], row_lds);
@@ -244,11 +243,11 @@ void flash_f32_kernel(Params p) {
         else dma16_m0<2 * kWave * 16>(src, voff[r], row_lds);
     };
     // the first byte of tile t's window in K or V
-    auto tile_src = [&](const float* base, int t) {
-        return (const char*)base + (size_t)win(k0 + t * BN) * (kDim * 4);
+    auto tile_src = [&](DmaSrc base, int t) {
+        return base + (size_t)win(k0 + t * BN) * (kDim * 4);
     };
     auto issue = [&](int ph) {  // phase 0 or 1 (the first tile's K or V) into buffer ph
-        const char* src = tile_src((ph & 1) ? Vs : Ks, 0);
+        const DmaSrc src = tile_src((ph & 1) ? Vs : Ks, 0);
 #pragma unroll
         for (int t = 0; t < CPW; ++t) dma_chunk(src, lds0 + 4u * (unsigned)(ph * BUF), t);
     };
@@ -263,7 +262,7 @@ void flash_f32_kernel(Params p) {
         // A block of 16 latents has a tile's shape: it comes by the same DMA,
         // into the third buffer, ahead of the first tile (latents past NL
         // repeat the last one).
-        const char* const qsrc = dma_base((const char*)(p.Q + ((size_t)b * p.NL + q0) * kDim));
+        const DmaSrc qsrc = dma_base(p.Q + ((size_t)b * p.NL + q0) * kDim);
 #pragma unroll
         for (int r = 0; r < CPW / ROW_CHUNKS; ++r) {
             const unsigned qoff =
@@ -430,8 +429,8 @@ void flash_f32_kernel(Params p) {
             // the next tile's K and V windows (the last tile re-reads its
             // own: phases past the end, loaded but never read)
             const int tnext = min(tile + 1, ntiles - 1);
-            const char* const ksrc = tile_src(Ks, tnext);
-            const char* const vsrc = tile_src(Vs, tnext);
+            const DmaSrc ksrc = tile_src(Ks, tnext);
+            const DmaSrc vsrc = tile_src(Vs, tnext);
 
             // ---------------- QK phase ----------------
             XATTN_STAMP(pc_b);

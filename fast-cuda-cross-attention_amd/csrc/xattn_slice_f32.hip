@@ -172,7 +172,7 @@ void slice_f32_kernel(Params p) {
     lds_char* const slice = L + w * 3 * SLICE;
     const unsigned slice0 = lds_u32(lds) + w * 3 * SLICE;
     auto ksrc = [&](int t) { return dma_base(Kb + (size_t)win(min(t, ntiles - 1)) * ROWB); };
-    auto dma_k = [&](const char* src, unsigned buf, int m) {
+    auto dma_k = [&](DmaSrc src, unsigned buf, int m) {
         dma16_m0<0>(src, goff[m], slice0 + buf + 1024 * m);
     };
     // operand read: lane (j, g) takes row j, piece 4 u + g
@@ -265,7 +265,7 @@ void slice_f32_kernel(Params p) {
         // Q comes through the third slice (latents past NL repeat the last),
         // with K(0), K(1) and V(0) behind it.
         {
-            const char* const qsrc = dma_base((const char*)(p.Q + ((size_t)b * p.NL + q0) * kDim));
+            const DmaSrc qsrc = dma_base(p.Q + ((size_t)b * p.NL + q0) * kDim);
             const int qlast = min(p.NL - q0, BM) - 1;
 #pragma unroll
             for (int m = 0; m < NCH; ++m) {
@@ -273,10 +273,10 @@ void slice_f32_kernel(Params p) {
                 dma16_m0<0>(qsrc, ROWB * min(r, qlast) + 4 * DW * w + 16 * (c ^ r),
                             slice0 + 2 * SLICE + 1024 * m);
             }
-            const char* const sk0 = ksrc(0);
+            const DmaSrc sk0 = ksrc(0);
 #pragma unroll
             for (int m = 0; m < NCH; ++m) dma_k(sk0, 0, m);
-            const char* const sk1 = ksrc(1);
+            const DmaSrc sk1 = ksrc(1);
 #pragma unroll
             for (int m = 0; m < NCH; ++m) dma_k(sk1, SLICE, m);
             const auto rv = rsrc(Vb, 0);
@@ -300,7 +300,7 @@ void slice_f32_kernel(Params p) {
         compiler_fence();
         // the first tile's scores and weights
         {
-            const char* const sk = ksrc(2);
+            const DmaSrc sk = ksrc(2);
             wait_vmcnt<24>();  // K(0)
 #pragma unroll
             for (int u = 0; u < KPF; ++u) read_k(0, u);
@@ -327,7 +327,7 @@ void slice_f32_kernel(Params p) {
             const unsigned kc = turn * SLICE, kn = (turn == 2 ? 0 : turn + 1) * SLICE;
             const unsigned kl = (turn == 0 ? 2 : turn - 1) * SLICE;
             const int xb = turn * (NW * 1024);
-            const char* const sk = ksrc(t + 2);
+            const DmaSrc sk = ksrc(t + 2);
 #pragma unroll
             for (int u = 0; u < NU; ++u) {
                 qk_group(u);
