@@ -682,17 +682,21 @@ void lse_combine_kernel(const float* __restrict__ po, const float* __restrict__ 
 int f32_row_blocks(int NL, int ds) { return (NL + f32::BM / ds - 1) / (f32::BM / ds); }
 
 #ifdef XATTN_PHASE_CLOCK
-// The fp32 kernel's stamps: [kClockBlocks][8][kClockFields] unsigned 64-bit
+// The fp32 kernels' stamps: [kClockBlocks][8][kClockFields] unsigned 64-bit
 // values (four wavefronts used).  Clear before a launch, read after.  0 on
 // success.
+unsigned long long* f32_phase_clock() {
+    void* ptr = nullptr;
+    if (hipGetSymbolAddress(&ptr, HIP_SYMBOL(f32::phase_clock)) != hipSuccess) return nullptr;
+    return (unsigned long long*)ptr;
+}
 extern "C" int xattn_phase_clock_read_f32(void* dst, size_t bytes) {
     const size_t n = bytes < sizeof(f32::phase_clock) ? bytes : sizeof(f32::phase_clock);
     return hipMemcpyFromSymbol(dst, HIP_SYMBOL(f32::phase_clock), n) == hipSuccess ? 0 : 1;
 }
 extern "C" int xattn_phase_clock_clear_f32(void) {
-    void* ptr = nullptr;
-    if (hipGetSymbolAddress(&ptr, HIP_SYMBOL(f32::phase_clock)) != hipSuccess) return 1;
-    if (hipMemset(ptr, 0, sizeof(f32::phase_clock)) != hipSuccess) return 1;
+    void* const ptr = f32_phase_clock();
+    if (!ptr || hipMemset(ptr, 0, sizeof(f32::phase_clock)) != hipSuccess) return 1;
     return hipDeviceSynchronize() == hipSuccess ? 0 : 1;
 }
 #endif

@@ -28,6 +28,10 @@ bool launch_flash_f32(int ds, const float* Q, const float* K, const float* V, fl
 bool launch_slice_f32(const float* Q, const float* K, const float* V, float* out, float* po,
                       float* pm, float* pl, int B, int NL, int NI, int S, int chunk,
                       hipStream_t stream);
+#ifdef XATTN_PHASE_CLOCK
+// Device address of the fp32 kernels' phase stamps, null where it cannot be had.
+unsigned long long* f32_phase_clock();
+#endif
 // The LSE merge of split partials into out; parts <= 0 takes
 // lse_combine_parts' column parts (1, 2 or 4 workgroups per row; any choice
 // gives bit-identical output).

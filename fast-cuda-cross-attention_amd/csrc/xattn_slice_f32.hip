@@ -65,6 +65,9 @@ struct Params {
     float* pm;
     float* pl;
     int B, NL, NI, S, chunk, row_blocks;
+#ifdef XATTN_PHASE_CLOCK
+    unsigned long long* clock;  // flash_f32_kernel's stamps, which this form fills in its place
+#endif
 };
 
 typedef __attribute__((address_space(3))) char lds_char;
@@ -98,6 +101,10 @@ void slice_f32_kernel(Params p) {
     constexpr int FLAG = XCH + 3 * NW * 1024;
     __shared__ __attribute__((aligned(16))) char lds[FLAG + 16];
 
+    XATTN_STAMP(clk_start);
+#ifdef XATTN_PHASE_CLOCK
+    const unsigned long long rt_start = __builtin_amdgcn_s_memrealtime();
+#endif
     const int item = xcd_remap(blockIdx.x, gridDim.x);
     const int rb = item % p.row_blocks;
     const int bs = item / p.row_blocks;
@@ -261,6 +268,9 @@ void slice_f32_kernel(Params p) {
     };
 #define PIN() __builtin_amdgcn_sched_barrier(0)
 
+    // first-phase sums are score phases, second-phase sums output products
+    // and the softmax after them
+    XATTN_CLOCK_DECL(clk_loop = 0, pc_wait = 0, pc_qk = 0, pc_pv = 0);
     for (;;) {  // passes over the key range; a second is rare
         // Q comes through the third slice (latents past NL repeat the last),
         // with K(0), K(1) and V(0) behind it.
@@ -298,6 +308,10 @@ void slice_f32_kernel(Params p) {
             qr[u] = lds_read<f4>(slice + 2 * SLICE + srd[u & 3] + 256 * (u >> 2));
         __builtin_amdgcn_s_waitcnt(0xC07F);  // read before the DMA of K(2) writes there
         compiler_fence();
+        XATTN_STAMP(pc_q);
+#ifdef XATTN_PHASE_CLOCK
+        if (clk_loop == 0) clk_loop = pc_q;
+#endif
         // the first tile's scores and weights
         {
             const DmaSrc sk = ksrc(2);
@@ -313,12 +327,18 @@ void slice_f32_kernel(Params p) {
                 PIN();
             }
             lds_write(xwr, s);
+            XATTN_STAMP(pc_c);
             lds_barrier();
+            XATTN_STAMP(pc_d);
             read_shares(0);
             wait_vmcnt<24>();  // K(1)
 #pragma unroll
             for (int u = 0; u < KPF; ++u) read_k(SLICE, u);
             softmax(0);
+            XATTN_STAMP(pc_e);
+            XATTN_CLOCK_ADD(pc_qk, pc_q, pc_c);
+            XATTN_CLOCK_ADD(pc_wait, pc_c, pc_d);
+            XATTN_CLOCK_ADD(pc_pv, pc_d, pc_e);
         }
         // Tile t's scores, then tile t - 1's output product, under whose MFMAs
         // the scores are exchanged.  K(t + 2) and V(t) are requested.
@@ -328,6 +348,7 @@ void slice_f32_kernel(Params p) {
             const unsigned kl = (turn == 0 ? 2 : turn - 1) * SLICE;
             const int xb = turn * (NW * 1024);
             const DmaSrc sk = ksrc(t + 2);
+            XATTN_STAMP(pc_a);
 #pragma unroll
             for (int u = 0; u < NU; ++u) {
                 qk_group(u);
@@ -337,6 +358,7 @@ void slice_f32_kernel(Params p) {
                 PIN();
             }
             lds_write(xwr + xb, s);
+            XATTN_STAMP(pc_b);
             const auto rv = rsrc(Vb, t);
 #pragma unroll
             for (int n = 0; n < 4 * NT; ++n) {
@@ -344,7 +366,11 @@ void slice_f32_kernel(Params p) {
                 PIN();
                 load_v(rv, n);
                 if (n == 4) {
+                    XATTN_STAMP(pc_c);
                     lds_barrier();
+                    XATTN_STAMP(pc_d);
+                    XATTN_CLOCK_ADD(pc_wait, pc_c, pc_d);
+                    XATTN_CLOCK_ADD(pc_pv, pc_d, pc_c);  // a wait, not the output product's time
                     read_shares(xb);
                 }
                 if (n == 8) wait_vmcnt<21>();  // K(t + 1)
@@ -352,6 +378,9 @@ void slice_f32_kernel(Params p) {
                 PIN();
             }
             softmax(t);
+            XATTN_STAMP(pc_e);
+            XATTN_CLOCK_ADD(pc_qk, pc_a, pc_b);
+            XATTN_CLOCK_ADD(pc_pv, pc_b, pc_e);
         };
         int t = 1;
         for (; t + 2 < ntiles; t += 3) {
@@ -361,8 +390,11 @@ void slice_f32_kernel(Params p) {
         }
         for (int turn = 1; t < ntiles; ++t, ++turn) tile(t, turn);
         // the last tile's output product
+        XATTN_STAMP(pc_l);
 #pragma unroll
         for (int n = 0; n < 4 * NT; ++n) pv_group(n);
+        XATTN_STAMP(pc_m);
+        XATTN_CLOCK_ADD(pc_pv, pc_l, pc_m);
         wait_vmcnt<0>();  // the re-reads of the last tile
 
         // Every wavefront raises the flag (if at all) before this barrier, so
@@ -378,6 +410,7 @@ void slice_f32_kernel(Params p) {
         bound = m_ref + tau_raw;
     }
 
+    XATTN_STAMP(clk_loop_end);
     // The latent's exact max and sum of weights over its four lanes.
     m_true = wave_max16_groups(m_true);
     lsum = wave_sum16_groups(lsum);
@@ -404,6 +437,15 @@ void slice_f32_kernel(Params p) {
         p.pm[pi] = m_true / sqrtf((float)kDim);
         p.pl[pi] = lsum * factor;
     }
+#ifdef XATTN_PHASE_CLOCK
+    XATTN_STAMP(clk_end);
+    const unsigned long long rt_end = __builtin_amdgcn_s_memrealtime();
+    if (lane == 0 && p.clock && blockIdx.x < (unsigned)kClockBlocks) {
+        unsigned long long* c = p.clock + ((size_t)blockIdx.x * 8 + w) * kClockFields;
+        c[0] = clk_start, c[1] = clk_loop, c[2] = clk_loop_end, c[3] = clk_end;
+        c[4] = rt_start, c[5] = rt_end, c[6] = pc_wait, c[7] = pc_qk, c[8] = pc_pv;
+    }
+#endif
 }
 
 }  // namespace f32s
@@ -415,6 +457,9 @@ bool launch_slice_f32(const float* Q, const float* K, const float* V, float* out
     p.Q = Q; p.K = K; p.V = V; p.out = out; p.po = po; p.pm = pm; p.pl = pl;
     p.B = B; p.NL = NL; p.NI = NI; p.S = S; p.chunk = chunk;
     p.row_blocks = (NL + f32s::BM - 1) / f32s::BM;
+#ifdef XATTN_PHASE_CLOCK
+    p.clock = f32_phase_clock();
+#endif
     const long long nblk = (long long)B * p.row_blocks * S;
     if (nblk <= 0) return true;
     if (nblk > 0x7fffffffLL) {

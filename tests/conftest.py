@@ -1,5 +1,9 @@
 import os
+import shlex
+import shutil
+import subprocess
 import sys
+from concurrent.futures import ThreadPoolExecutor
 
 import numpy as np
 import pytest
@@ -31,6 +35,45 @@ def cw():
 def oracle():
     import xattn_oracle
     return xattn_oracle
+
+
+HIPCC = "/opt/rocm/bin/hipcc"
+
+
+def build_recipes():
+    """(source, library, compiler arguments) of every HIP source of kernels.so
+    and of kernels_phaseclock.so, as the Makefile compiles them."""
+    out = []
+    for target in ("kernels.so", "kernels_phaseclock.so"):
+        lines = subprocess.run(["make", "-n", "-B", target], cwd=PKG, check=True,
+                               capture_output=True, text=True).stdout.splitlines()
+        for args in map(shlex.split, lines):
+            if "-c" in args:
+                at = args.index("-c")
+                out.append((args[at + 1], target,
+                            [a for a in args[:at] if a != "-o" and not a.endswith(".o")]))
+    return out
+
+
+def assemble(source, recipe, target):
+    """Compiles a source to AMD assembly with a recipe's arguments."""
+    return subprocess.run([*recipe, "-S", "--cuda-device-only", "-w", source, "-o", str(target)],
+                          cwd=PKG, capture_output=True, text=True)
+
+
+@pytest.fixture(scope="session")
+def device_asm(tmp_path_factory):
+    """{(source, library): AMD assembly} of both libraries' sources."""
+    if not shutil.which(HIPCC):
+        pytest.skip("hipcc not found")
+    folder, recipes = tmp_path_factory.mktemp("asm"), build_recipes()
+    targets = [folder / f"{i}.s" for i in range(len(recipes))]
+    with ThreadPoolExecutor(min(8, os.cpu_count() or 1)) as pool:
+        runs = list(pool.map(lambda r, t: assemble(r[0], r[2], t), recipes, targets))
+    for run in runs:
+        assert run.returncode == 0, run.stderr
+    return {(os.path.basename(source), library): target.read_text()
+            for (source, library, _), target in zip(recipes, targets)}
 
 
 def fp32_gate(out, ref, atol=1e-4, rtol=1e-3):

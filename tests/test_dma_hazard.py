@@ -9,18 +9,13 @@ maker waits; these tests compile every source the way the Makefile does, look
 the AMD assembly over for such a pair, and need no GPU.
 """
 
-import os
 import re
-import shlex
 import shutil
-import subprocess
-from concurrent.futures import ThreadPoolExecutor
 
 import pytest
 
-from conftest import PKG
+from conftest import HIPCC, assemble, build_recipes
 
-HIPCC = "/opt/rocm/bin/hipcc"
 WAIT_STATES = 5
 pytestmark = pytest.mark.skipif(not shutil.which(HIPCC), reason="hipcc not found")
 
@@ -91,26 +86,6 @@ def hazards(asm):
     return found
 
 
-def _recipes():
-    """{source: compiler arguments up to -c} of both libraries' builds."""
-    lines = subprocess.run(["make", "-n", "-B", "all", "phaseclock"], cwd=PKG, check=True,
-                           capture_output=True, text=True).stdout.splitlines()
-    out = []
-    for line in lines:
-        args = shlex.split(line)
-        if "-c" in args:
-            at = args.index("-c")
-            out.append((args[at + 1], [a for a in args[:at] + args[at + 2:]
-                                       if a != "-o" and not a.endswith(".o")]))
-    return out
-
-
-def _assemble(source, recipe, target):
-    args = [a for a in recipe if a != "-c"] + ["-S", "--cuda-device-only", "-w", source,
-                                               "-o", str(target)]
-    return subprocess.run(args, cwd=PKG, capture_output=True, text=True)
-
-
 def test_the_scan_finds_a_pair_and_counts_its_wait_states():
     def kernel(*between):
         return "\n".join(["k:", "v_readfirstlane_b32 s5, v1", *between,
@@ -127,19 +102,11 @@ def test_the_scan_finds_a_pair_and_counts_its_wait_states():
     assert hazards("\n".join(loop)) == []
 
 
-def test_the_kernels_keep_the_wait_states(tmp_path):
-    recipes = _recipes()
-    assert len(recipes) == 10, [r[0] for r in recipes]  # five sources, two libraries
-    targets = [tmp_path / f"{i}.s" for i in range(len(recipes))]
-    with ThreadPoolExecutor(min(8, os.cpu_count() or 1)) as pool:
-        runs = list(pool.map(lambda r, t: _assemble(*r, t), recipes, targets))
-    dmas = 0
-    for (source, _), run, target in zip(recipes, runs, targets):
-        assert run.returncode == 0, run.stderr
-        asm = target.read_text()
-        dmas += asm.count("global_load_lds")
-        assert hazards(asm) == [], source
-    assert dmas > 100
+def test_the_kernels_keep_the_wait_states(device_asm):
+    assert len(device_asm) == 10, list(device_asm)  # five sources, two libraries
+    assert sum(asm.count("global_load_lds") for asm in device_asm.values()) > 100
+    found = {which: hazards(asm) for which, asm in device_asm.items() if hazards(asm)}
+    assert not found, found
 
 
 PROBE = """
@@ -160,14 +127,14 @@ __global__ void probe(const char* a, int stride, float* out) {
 def test_the_dma_takes_no_base_that_was_not_waited_for(tmp_path, dma):
     """The tightest code a kernel can write: refused with a plain pointer, and
     with the waiting base no pair in the assembly."""
-    recipe = next(r for s, r in _recipes() if "flash_f16" in s)
+    recipe = next(r for s, _, r in build_recipes() if "flash_f16" in s)
 
     def probe(name, base):
         source = tmp_path / f"{name}.hip"
         source.write_text(PROBE.replace(
             "BODY", f"{dma}({base}, 16u * (threadIdx.x & 63), lds_u32(lds));"))
         target = tmp_path / f"{name}.s"
-        return _assemble(str(source), recipe, target), target
+        return assemble(str(source), recipe, target), target
 
     run, target = probe("plain", "uniform_ptr(p)")
     assert run.returncode != 0, "\n".join(hazards(target.read_text()))
