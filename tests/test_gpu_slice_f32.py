@@ -19,13 +19,21 @@ def test_tile_counts(cw, oracle, nl, ni):
     fp32_gate(out, oracle.attention_f64(q, k, v))
 
 
-@pytest.mark.parametrize("rest", [1, 15, 16, 17, 48])
-def test_short_last_split(cw, oracle, rest):
-    """145 splits of 144 keys, the last of which has ``rest``; the partials
-    against the oracle's."""
-    ni, splits = 144 * 144 + rest, 145
-    q, k, v = oracle.make_inputs(1, 17, ni, 768, seed=rest)
-    out, (po, pm, pl) = cw.splitk_partials(q, k, v, 1, 17, ni, 768, splits)
+@pytest.mark.parametrize("nl, splits, keys, rest",
+                         [(16, 145, 144, rest) for rest in (1, 15, 16, 17, 48)]
+                         + [(17, 128, 129, rest) for rest in (2, 15, 16, 17, 48)])
+def test_short_last_split(cw, oracle, nl, splits, keys, rest):
+    """Splits of 9 tiles, the last of which has ``rest`` keys only (its window
+    clamped or shifted, its look-ahead past its end), with a whole latent block
+    and a block of one latent; the partials against the oracle's.  The counts
+    are ones that the planner gives 16 latents per workgroup."""
+    ni = (splits - 1) * keys + rest
+    assert -(-ni // splits) == keys
+    cu, _ = cw.device_info()
+    if cu == 256:
+        assert cw.lib.xattn_f32_split_latents(1, nl, ni, splits, cu) == 16
+    q, k, v = oracle.make_inputs(1, nl, ni, 768, seed=rest)
+    out, (po, pm, pl) = cw.splitk_partials(q, k, v, 1, nl, ni, 768, splits)
     fp32_gate(out, oracle.attention_f64(q, k, v))
     s = (q[0].astype(np.float64) @ k[0, -rest:].astype(np.float64).T) / np.sqrt(768.0)
     m = s.max(axis=1)
