@@ -46,7 +46,8 @@ def _kernels(tmp_path):
         # Within a kernel's entry the keys are sorted: its arguments' .name
         # fields come first, then the kernel's own .name, then
         # .private_segment_fixed_size; .group_segment_fixed_size precedes both.
-        name, group = None, None
+        # The spill counts come after those.
+        name, group, last = None, None, None
         for line in notes.splitlines():
             m = re.match(r"\s*-?\s*\.(\w+):\s+(\S+)", line)
             if not m:
@@ -57,8 +58,10 @@ def _kernels(tmp_path):
             elif key == "name":
                 name = val
             elif key == "private_segment_fixed_size" and name is not None:
-                out[name] = {"private": int(val), "group": group}
+                out[name] = last = {"private": int(val), "group": group}
                 name, group = None, None
+            elif key in ("sgpr_spill_count", "vgpr_spill_count"):
+                last[key] = int(val)
     return out
 
 
@@ -75,16 +78,37 @@ def kernels(tmp_path_factory):
 def test_every_instantiation_is_present(kernels):
     names = list(kernels)
     assert sum("flash_f32_kernel" in n for n in names) == 6   # {split, full} x DS {1, 2, 4}
+    assert sum("slice_f32_kernel" in n for n in names) == 2   # {split, full}
     assert sum("flash16_kernel" in n for n in names) == 12    # {fp16, bf16} x split x 3 forms
     assert sum("lse_combine_kernel" in n for n in names) == 4
     assert any("naive_kernel" in n for n in names)
 
 
+HOT = ("flash_f32_kernel", "slice_f32_kernel", "flash16_kernel", "lse_combine_kernel")
+
+
 def test_hot_kernels_do_not_spill(kernels):
-    hot = {n: k for n, k in kernels.items()
-           if any(s in n for s in ("flash_f32_kernel", "flash16_kernel", "lse_combine_kernel"))}
+    hot = {n: k for n, k in kernels.items() if any(s in n for s in HOT)}
     spilled = {n: k["private"] for n, k in hot.items() if k["private"] != 0}
     assert not spilled, f"kernels with a scratch segment (bytes per lane): {spilled}"
+    vgprs = {n: k["vgpr_spill_count"] for n, k in hot.items() if k["vgpr_spill_count"] != 0}
+    assert not vgprs, f"kernels that spill vector registers: {vgprs}"
+
+
+def test_scalar_spills_stay_outside_the_key_loops(kernels, device_asm):
+    """A scalar register may be kept in a lane of a vector register, as the split
+    slice form does with the epilogue's addresses (13), but not between a
+    kernel's first and last MFMA: there each move is a vector instruction that
+    the matrix pipe waits for."""
+    bodies = {m[1]: m[2] for (_, library), asm in device_asm.items() if library == "kernels.so"
+              for m in re.finditer(r"^(_Z\w+):.*?\n(.*?)^\.Lfunc_end", asm, re.S | re.M)}
+    flash = [n for n in kernels if "flash" in n or "slice" in n]
+    assert len(flash) == 6 + 2 + 12
+    for name in flash:
+        ops = [line.split()[0] for line in bodies[name].splitlines() if line.startswith("\tv_")]
+        mfma = [i for i, op in enumerate(ops) if op.startswith("v_mfma")]
+        moved = [op for op in ops[mfma[0]:mfma[-1]] if op in ("v_readlane_b32", "v_writelane_b32")]
+        assert not moved, (name, kernels[name]["sgpr_spill_count"], moved)
 
 
 def test_lds_fits_one_cu(kernels):
