@@ -56,3 +56,25 @@ def test_scores_that_outgrow_the_first_tile(cw, oracle):
         score_err = 2.0 ** -24 * np.max(np.abs(q[0]) @ np.abs(k[0]).T) / np.sqrt(768.0)
         fp32_gate(out, oracle.attention_f64(q, k, v),
                   atol=float(2.0 * score_err * np.max(np.abs(v))))
+
+
+@pytest.mark.parametrize("splits", [1, 2])
+@pytest.mark.parametrize("key", [5, 77, 149, 299])
+def test_nan_stays_where_the_reference_puts_it(cw, oracle, key, splits):
+    """As the fp32 tests' case of that name, over ranges that take this form
+    (19 tiles of 16, or two splits of 10 and 9): a NaN in one batch element's K
+    makes that element's whole output NaN, in its V only one column; every
+    other value matches.  The key sits in the first tile, in the loop, in the
+    last tile of a split and in a partial last tile, whose window repeats keys
+    of the tile before."""
+    b, nl, ni = 3, 17, 300
+    for where in ("K", "V"):
+        q, k, v = oracle.make_inputs(b, nl, ni, 768, seed=79)
+        (k if where == "K" else v)[1, key, 5] = np.nan
+        ref = oracle.attention_f64(q, k, v)
+        nan = np.isnan(ref)
+        assert nan[1].any() and not nan[[0, 2]].any()
+        out, _, _ = cw.benchmark_plan_events(q, k, v, b, nl, ni, 768, 16, splits, warmup=1,
+                                             iters=0)
+        assert np.array_equal(np.isnan(out), nan), f"NaN in {where}: NaN pattern"
+        fp32_gate(np.where(nan, 0.0, out), np.where(nan, 0.0, ref))
