@@ -268,9 +268,10 @@ void slice_f32_kernel(Params p) {
     };
 #define PIN() __builtin_amdgcn_sched_barrier(0)
 
-    // first-phase sums are score phases, second-phase sums output products
-    // and the softmax after them
-    XATTN_CLOCK_DECL(clk_loop = 0, pc_wait = 0, pc_qk = 0, pc_pv = 0);
+    // The first phase is the scores; the second, all the rest of the loop
+    // (output products, softmax), is the loop's time less the others': a sum
+    // of its own and the stamps for it cost 90 cycles per tile more.
+    XATTN_CLOCK_DECL(clk_loop = 0, pc_wait = 0, pc_qk = 0);
     for (;;) {  // passes over the key range; a second is rare
         // Q comes through the third slice (latents past NL repeat the last),
         // with K(0), K(1) and V(0) behind it.
@@ -335,10 +336,8 @@ void slice_f32_kernel(Params p) {
 #pragma unroll
             for (int u = 0; u < KPF; ++u) read_k(SLICE, u);
             softmax(0);
-            XATTN_STAMP(pc_e);
             XATTN_CLOCK_ADD(pc_qk, pc_q, pc_c);
             XATTN_CLOCK_ADD(pc_wait, pc_c, pc_d);
-            XATTN_CLOCK_ADD(pc_pv, pc_d, pc_e);
         }
         // Tile t's scores, then tile t - 1's output product, under whose MFMAs
         // the scores are exchanged.  K(t + 2) and V(t) are requested.
@@ -359,6 +358,7 @@ void slice_f32_kernel(Params p) {
             }
             lds_write(xwr + xb, s);
             XATTN_STAMP(pc_b);
+            XATTN_CLOCK_ADD(pc_qk, pc_a, pc_b);
             const auto rv = rsrc(Vb, t);
 #pragma unroll
             for (int n = 0; n < 4 * NT; ++n) {
@@ -370,7 +370,6 @@ void slice_f32_kernel(Params p) {
                     lds_barrier();
                     XATTN_STAMP(pc_d);
                     XATTN_CLOCK_ADD(pc_wait, pc_c, pc_d);
-                    XATTN_CLOCK_ADD(pc_pv, pc_d, pc_c);  // a wait, not the output product's time
                     read_shares(xb);
                 }
                 if (n == 8) wait_vmcnt<21>();  // K(t + 1)
@@ -378,9 +377,6 @@ void slice_f32_kernel(Params p) {
                 PIN();
             }
             softmax(t);
-            XATTN_STAMP(pc_e);
-            XATTN_CLOCK_ADD(pc_qk, pc_a, pc_b);
-            XATTN_CLOCK_ADD(pc_pv, pc_b, pc_e);
         };
         int t = 1;
         for (; t + 2 < ntiles; t += 3) {
@@ -390,11 +386,8 @@ void slice_f32_kernel(Params p) {
         }
         for (int turn = 1; t < ntiles; ++t, ++turn) tile(t, turn);
         // the last tile's output product
-        XATTN_STAMP(pc_l);
 #pragma unroll
         for (int n = 0; n < 4 * NT; ++n) pv_group(n);
-        XATTN_STAMP(pc_m);
-        XATTN_CLOCK_ADD(pc_pv, pc_l, pc_m);
         wait_vmcnt<0>();  // the re-reads of the last tile
 
         // Every wavefront raises the flag (if at all) before this barrier, so
@@ -443,7 +436,8 @@ void slice_f32_kernel(Params p) {
     if (lane == 0 && p.clock && blockIdx.x < (unsigned)kClockBlocks) {
         unsigned long long* c = p.clock + ((size_t)blockIdx.x * 8 + w) * kClockFields;
         c[0] = clk_start, c[1] = clk_loop, c[2] = clk_loop_end, c[3] = clk_end;
-        c[4] = rt_start, c[5] = rt_end, c[6] = pc_wait, c[7] = pc_qk, c[8] = pc_pv;
+        c[4] = rt_start, c[5] = rt_end, c[6] = pc_wait, c[7] = pc_qk;
+        c[8] = clk_loop_end - clk_loop - pc_wait - pc_qk;
     }
 #endif
 }
