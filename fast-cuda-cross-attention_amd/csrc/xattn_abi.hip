@@ -342,10 +342,13 @@ int plan_splits(int B, int NL, int NI, int cu, int bm, int tile) {
 // often per FLOP), plus 0.68 µs per round of workgroups; a split launch adds
 // the LSE merge, 10.67 µs + 0.36 µs per MB of partials written and read back,
 // + 0.08 µs per split while there are fewer merge rows (B * N_latent) than
-// CUs.  Its choice is the fastest timed plan at 27 of the 31 shapes, 0.48 %
-// slower on average and 4.4 % at worst.  Ranges of nine or more tiles have since
-// got faster at 16 latents (1.40-1.45 µs per tile, xattn_slice_f32.hip), which
-// the fit does not hold.
+// CUs.  At 16 latents the fit is of the column-split form; ranges of nine or
+// more tiles now take 1.46-1.51 µs per tile (xattn_slice_f32.hip), so 16 latents
+// are chosen there only where they win at 1.72.  With today's kernels, calls
+// issued back to back, its choice is 0.3 % slower than the best timed plan on
+// average over 32 shapes of that range (8.8 % at worst, B=1 N_latent=128
+// N_input=784) and 0.5 % over 45 drawn ones (6.7 %, B=30 N_latent=658
+// N_input=975).
 static double f32_cost(int B, int NL, int cu, int ds, long long S, long long ct) {
     const double tile_us = ds == 1 ? 5.620 : ds == 2 ? 2.986 : 1.716;
     const long long W = (long long)B * f32_row_blocks(NL, ds) * S;

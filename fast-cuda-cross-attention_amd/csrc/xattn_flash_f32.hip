@@ -720,9 +720,13 @@ bool launch_flash_f32(int ds, const float* Q, const float* K, const float* V, fl
     }
     if (ds == 4) {
         // 16-latent workgroups: the sliced form for longer key ranges.  Its
-        // loop is 7 % faster per tile, its first tiles cost more: ranges of 7
-        // tiles measured 1.2 % slower with it, of 11 / 16 / 49 tiles 3.5 / 4.2
-        // / 6.8 % faster (B=1 NL=512, B=3 NL=197, B=1 NL=256, B=8 NL=512).
+        // loop is 7-8 % faster per tile, its first tiles cost more.  Over nine
+        // launches (64 to 512 workgroups, split and unsplit, whole and partial
+        // last tiles) it measured, in time of the column-split form over its
+        // own, 0.982-0.998 at 5 tiles, 0.996-1.012 at 7, 0.998-1.018 at 8,
+        // 1.003-1.021 at 9, 1.004-1.027 at 10 and 1.012-1.036 at 12; B=8
+        // NL=512 NI=784 (49 tiles) 1.064.  Nine is the shortest range at which
+        // no launch was slower.
         constexpr int kSliceMinTiles = 9;
         const int keys = po ? (chunk < NI ? chunk : NI) : NI;
         if ((keys + f32::BN - 1) / f32::BN >= kSliceMinTiles)

@@ -18,17 +18,22 @@
 //   * no wavefront reads another's columns, so tiles need no barrier: K comes
 //     by DMA into the wavefront's own ring of three LDS slices, V by loads
 //     straight into the operand's registers (its lanes lie on consecutive
-//     bytes), each a tile or more ahead;
+//     bytes).  V(t) is requested a whole tile before its MFMAs.  K(t + 2) is
+//     requested one and a half tiles before its first read, but has about half
+//     a tile to arrive: the compiler, which counts the V loads and not the
+//     DMA, waits before each output group for vmcnt(11), and the counter is in
+//     order, so group n of V(t - 1) also waits for piece n of K(t + 2),
+//     requested 48 MFMAs earlier;
 //   * tile t's scores come before tile t - 1's output product, so the one
-//     barrier of a tile, the exchange's round trip through LDS and the MFMA
-//     results' latency pass under MFMAs;
+//     barrier of a tile and the exchange's reads pass under MFMAs (the write
+//     of the shares does not: it waits for the last score MFMA's result);
 //   * the tile loop is unrolled over the three slices, so LDS addresses are
 //     registers set up once plus immediates, and the softmax is one run of
 //     vector instructions per tile.
-// Per tile 3,348 cycles at 2.4 GHz with 256 workgroups and 3,484 with 64 (1.395
-// / 1.452 us) against 3,603 / 3,791 (1.501 / 1.579 us) of the column-split form
-// of flash_f32_kernel, whose wavefronts share row-wise tiles through two
-// barriers per tile; without the softmax it takes 3,117 / 3,185.  B=8 NL=512
+// Per tile 1.46 us with 64 workgroups (3,490 cycles at 2.40 GHz) and 1.49-1.51
+// with 256, in the same cycles at the lower clock of a full device, against
+// 1.59 and 1.61 us of the column-split form of flash_f32_kernel, whose
+// wavefronts share row-wise tiles through two barriers per tile.  B=8 NL=512
 // NI=784: 79.0 against 84.4 us per call.  Measured and not kept: a tile's
 // weights dealt to the four wavefronts (a quarter of the vector instructions,
 // one more exchange: the same time); K through registers and ds_write
@@ -372,7 +377,9 @@ void slice_f32_kernel(Params p) {
                     XATTN_CLOCK_ADD(pc_wait, pc_c, pc_d);
                     read_shares(xb);
                 }
-                if (n == 8) wait_vmcnt<21>();  // K(t + 1)
+                // K(t + 1): all that its reads need (the V waits in front ask
+                // for more today, but only as the compiler places them)
+                if (n == 8) wait_vmcnt<21>();
                 if (n >= 8) read_k(kn, n - 8);
                 PIN();
             }
