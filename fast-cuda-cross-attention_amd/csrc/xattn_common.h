@@ -132,8 +132,14 @@ struct DmaSrc {
 };
 __device__ inline DmaSrc dma_base(const void* p) {
     const char* u = uniform_ptr((const char*)p);
-    asm volatile("s_nop 4" : "+s"(u));
+    asm("s_nop 4" : "+s"(u));
     return DmaSrc{u};
+}
+// Two bases behind one wait (an s_nop 4 holds a wavefront for about 20 cycles).
+__device__ inline void dma_base2(const void* p, const void* q, DmaSrc& a, DmaSrc& b) {
+    a.p = uniform_ptr((const char*)p);
+    b.p = uniform_ptr((const char*)q);
+    asm("s_nop 4" : "+s"(a.p), "+s"(b.p));
 }
 
 // 16-byte global -> LDS DMA for one lane.  The 64 lanes of the wave land at

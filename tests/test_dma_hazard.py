@@ -115,6 +115,8 @@ using namespace xattn;
 __global__ void probe(const char* a, int stride, float* out) {
     __shared__ __attribute__((aligned(16))) char lds[4096];
     const char* p = a + (size_t)(threadIdx.x >> 6) * stride;
+    struct { DmaSrc a, b; } two;
+    dma_base2(a, p, two.a, two.b);
     BODY
     wait_vmcnt<0>();
     lds_barrier();
@@ -139,8 +141,9 @@ def test_the_dma_takes_no_base_that_was_not_waited_for(tmp_path, dma):
     run, target = probe("plain", "uniform_ptr(p)")
     assert run.returncode != 0, "\n".join(hazards(target.read_text()))
     assert "DmaSrc" in run.stderr
-    run, target = probe("waited", "dma_base(p)")
-    assert run.returncode == 0, run.stderr
-    asm = target.read_text()
-    assert "v_readfirstlane" in asm and "global_load_lds" in asm
-    assert hazards(asm) == []
+    for name, base in (("one", "dma_base(p)"), ("two", "two.b")):
+        run, target = probe(name, base)
+        assert run.returncode == 0, run.stderr
+        asm = target.read_text()
+        assert "v_readfirstlane" in asm and "global_load_lds" in asm
+        assert hazards(asm) == []
